@@ -187,6 +187,26 @@ int sph_get_timing(const sph_t* h, sph_timing_t* out);
  * (default), 0 = plain launches, one kernel per stage. */
 int sph_set_graph(sph_t* h, int on);
 
+/* How steps run where the search and force kernels are left automatic and
+ * steps are not plain launches: SPH_PATH_AUTO (the default) as sph_set_search
+ * describes, SPH_PATH_CHAIN as a chain of like launches with neighbour lists
+ * whatever the size, SPH_PATH_STAGES as the graph of one kernel per stage,
+ * its search chosen by timing.  All give the same bits. */
+#define SPH_PATH_AUTO 0
+#define SPH_PATH_CHAIN 1
+#define SPH_PATH_STAGES 2
+int sph_set_path(sph_t* h, int path);
+
+/* What ran since the handle was opened, the autotuner's trial steps left out
+ * (an adjoint's recomputed steps count): steps as a chain and as stages, the
+ * chain's launches (those that found no work included), and the lanes that a
+ * chain of this handle takes for a sphere (4 or 1). */
+typedef struct sph_path {
+    uint64_t chain_steps, stage_steps, chain_launches;
+    uint32_t lanes;
+} sph_path_t;
+int sph_get_path(const sph_t* h, sph_path_t* out);
+
 /* Cells per contact-search block (tile_x along x, tile_y along y); 0, 0
  * restores the automatic choice made at open from the cell occupancy. */
 int sph_set_tile(sph_t* h, uint32_t tile_x, uint32_t tile_y);
@@ -352,11 +372,14 @@ int sph_ens_info(const sph_ens_t* e, sph_ens_info_t* out);
  * the next sph_ens_step the autotuner times the row, half-shell and list
  * kernels and then 64, 128 and 256 threads per block for the search and
  * force kernels, on ordinary steps, and keeps the fastest), 2, 4 or 5 (1 and
- * 3 walk one grid and are refused); graph capture; per-kernel profiling. */
+ * 3 walk one grid and are refused); graph capture; how steps run
+ * (sph_set_path); per-kernel profiling. */
 int sph_ens_set_precision(sph_ens_t* e, int precision);
 int sph_ens_set_search(sph_ens_t* e, int mode);
 int sph_ens_set_blocks(sph_ens_t* e, uint32_t force_block, uint32_t search_block);
 int sph_ens_set_graph(sph_ens_t* e, int on);
+int sph_ens_set_path(sph_ens_t* e, int path);
+int sph_ens_get_path(const sph_ens_t* e, sph_path_t* out);
 int sph_ens_set_profiling(sph_ens_t* e, int on);
 int sph_ens_get_timing(const sph_ens_t* e, sph_timing_t* out);
 

@@ -707,6 +707,7 @@ void run_one(sph_dem* h, const StepHooks* hooks) {
     h->own_cur ^= 1;
     h->hs.t_cur += h->hs.dt;
     ++h->steps_done;
+    ++h->ran.stage_steps;
 }
 
 }  // namespace

@@ -1078,15 +1078,17 @@ int sph::restore_state(sph_dem* h, const Checkpoint& c) {
 // Steps between two readings of the error flags.
 constexpr uint64_t STEP_CHUNK = 512;
 
-// A handle whose kernels the caller left to it.
+// A handle whose kernels the caller left to it, and that may step as a chain.
 static bool automatic(const sph_dem* h) {
-    return h->force_auto && (h->search_auto || (h->members.empty() && h->hs.contactmodel == 1));
+    return h->path != SPH_PATH_STAGES && h->force_auto && (h->search_auto || (h->members.empty() && h->hs.contactmodel == 1));
 }
 
 // ... whose steps are a chain of launches whatever a timing would say: small
-// enough for four lanes a sphere, or without a contact search to choose.
+// enough for four lanes a sphere, or without a contact search to choose, or at
+// the caller's wish.
 static bool chain_only(const sph_dem* h) {
-    return automatic(h) && h->members.empty() && (h->hs.np <= sph::QUAD_NP || h->hs.contactmodel == 1);
+    return automatic(h) && (h->path == SPH_PATH_CHAIN ||
+                            (h->members.empty() && (h->hs.np <= sph::QUAD_NP || h->hs.contactmodel == 1)));
 }
 
 bool sph::chained(const sph_dem* h) {
@@ -1117,6 +1119,7 @@ int stage_steps(sph_dem* h, uint64_t n) {
         h->own_cur ^= 1;
         h->hs.t_cur += h->hs.dt;
         ++h->steps_done;
+        ++h->ran.stage_steps;
         if ((i + 1) % STEP_CHUNK == 0 && i + 1 < n) {
             if ((rc = check_flags(h))) {
                 sph::launch_tail(sph::step_view(h, last), h->stream);
@@ -1185,6 +1188,7 @@ int sph::autotune(sph_dem* h) {
     }
     if (!tune_steps(h) || (h->tuned && h->steps_since_tune < 4096)) return SPH_OK;
     Checkpoint c;
+    const sph_path_t ran = h->ran;
     int rc;
     if ((rc = save_state(h, c))) return rc;
     // a simulation error inside the trial steps (the state blowing up within
@@ -1195,6 +1199,7 @@ int sph::autotune(sph_dem* h) {
     if (rc == SPH_E_HIP) return rc;
     h->tuned = true;
     h->steps_since_tune = 0;
+    h->ran = ran;
     destroy_graph(h);
     if ((rc = restore_state(h, c))) return rc;
     HIP_TRY(hipStreamSynchronize(h->stream));
@@ -1260,6 +1265,8 @@ int sph::chain_steps(sph_dem* h, uint32_t m, const Recording* rec) {
     if (m & 1) h->own_cur ^= 1;
     for (uint32_t k = 0; k < m; ++k) h->hs.t_cur += h->hs.dt;
     h->steps_done += m;
+    h->ran.chain_steps += m;
+    h->ran.chain_launches += l;
     return SPH_OK;
 }
 
@@ -1281,6 +1288,7 @@ int run_steps(sph_dem* h, uint64_t n) {
             t.search_ms += ms[3]; t.force_ms += ms[4]; t.walls_ms += ms[5];
             h->hs.t_cur += h->hs.dt;
             ++h->steps_done;
+            ++h->ran.stage_steps;
         }
         t.contact_ms = t.search_ms + t.force_ms;
         t.total_ms = t.bonds_ms + t.cellid_ms + t.sort_ms + t.reorder_ms + t.contact_ms + t.walls_ms;
@@ -1548,6 +1556,7 @@ int sph_readbin(sph_t* h, const char* path) {
     rc = open_common(t, h->verbosity, h->check_vals);
     if (!rc) {
         t->use_graph = h->use_graph;
+        t->path = h->path;
         t->search_auto = h->search_auto && t->hs.contactmodel != 1;
         t->profiling = h->profiling;
         if (t->d.search_mode == 5) request_list_rebuild(t);
@@ -1957,6 +1966,21 @@ int sph_set_graph(sph_t* h, int on) {
     return SPH_OK;
 }
 
+int sph_set_path(sph_t* h, int path) {
+    if (!h || path < SPH_PATH_AUTO || path > SPH_PATH_STAGES) return SPH_E_INVALID;
+    h->path = path;
+    h->tuned = false;
+    destroy_graph(h);
+    return SPH_OK;
+}
+
+int sph_get_path(const sph_t* h, sph_path_t* out) {
+    if (!h || !out) return SPH_E_INVALID;
+    *out = h->ran;
+    out->lanes = h->members.empty() && h->hs.np <= sph::QUAD_NP ? 4u : 1u;
+    return SPH_OK;
+}
+
 int sph_bandwidth_probe(uint64_t bytes, int reps, double* gbs) {
     if (bytes < 64 || reps < 1 || !gbs) return SPH_E_INVALID;
     const uint64_t n = bytes / 32;
@@ -2356,6 +2380,8 @@ int sph_ens_set_blocks(sph_ens_t* e, uint32_t force_block, uint32_t search_block
 }
 
 int sph_ens_set_graph(sph_ens_t* e, int on) { return e ? sph_set_graph(e->h, on) : SPH_E_INVALID; }
+int sph_ens_set_path(sph_ens_t* e, int path) { return e ? sph_set_path(e->h, path) : SPH_E_INVALID; }
+int sph_ens_get_path(const sph_ens_t* e, sph_path_t* out) { return e ? sph_get_path(e->h, out) : SPH_E_INVALID; }
 int sph_ens_set_profiling(sph_ens_t* e, int on) { return e ? sph_set_profiling(e->h, on) : SPH_E_INVALID; }
 int sph_ens_get_timing(const sph_ens_t* e, sph_timing_t* out) { return e ? sph_get_timing(e->h, out) : SPH_E_INVALID; }
 

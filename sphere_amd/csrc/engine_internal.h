@@ -48,6 +48,8 @@ struct sph_dem {
     bool force_auto = true;  // k_force variant chosen by timing (sph_set_force_kernel 0)
     uint64_t steps_since_tune = 0;
     bool tuned = false;
+    int path = SPH_PATH_AUTO;  // sph_set_path
+    sph_path_t ran{};          // what ran (lanes unused)
     bool as_chain = true;  // with lists: a chain of launches (by timing, where that is a choice), or the graph of stages
     // checkpoints, tape and adjoint buffers of sph_adjoint_* (adjoint.hip)
     std::unique_ptr<sph::AdjointState, void (*)(sph::AdjointState*)> adj{nullptr, nullptr};

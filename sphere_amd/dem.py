@@ -40,6 +40,9 @@ SPH_E_UNSUPPORTED = -8
 PREC_FP64 = 0
 PREC_MIXED = 1
 
+# how steps run (sph_set_path)
+PATHS = {"auto": 0, "chain": 1, "stages": 2}
+
 FIELDS: Dict[str, int] = {
     "x": 0, "vel": 1, "angvel": 2, "force": 3, "torque": 4, "angpos": 5,
     "xysum": 6, "vel0": 7, "angvel0": 8, "es_dot": 9, "es": 10, "ev_dot": 11,
@@ -111,6 +114,11 @@ class SphTiming(C.Structure):
                 ("list_builds", C.c_uint32)]
 
 
+class SphPath(C.Structure):
+    _fields_ = [("chain_steps", C.c_uint64), ("stage_steps", C.c_uint64), ("chain_launches", C.c_uint64),
+                ("lanes", C.c_uint32)]
+
+
 class SphEnsInfo(C.Structure):
     _fields_ = [("members", C.c_uint32), ("np", C.c_uint64), ("ncells", C.c_uint64), ("steps_done", C.c_uint64),
                 ("cell_factor", C.c_double), ("tuned_ms", C.c_double * 4), ("search_mode", C.c_int32),
@@ -137,6 +145,8 @@ EXPORTS = {
     "sph_set_profiling": (C.c_int, [C.c_void_p, C.c_int]),
     "sph_get_timing": (C.c_int, [C.c_void_p, C.POINTER(SphTiming)]),
     "sph_set_graph": (C.c_int, [C.c_void_p, C.c_int]),
+    "sph_set_path": (C.c_int, [C.c_void_p, C.c_int]),
+    "sph_get_path": (C.c_int, [C.c_void_p, C.POINTER(SphPath)]),
     "sph_set_tile": (C.c_int, [C.c_void_p, C.c_uint32, C.c_uint32]),
     "sph_set_search": (C.c_int, [C.c_void_p, C.c_int]),
     "sph_set_force_kernel": (C.c_int, [C.c_void_p, C.c_int]),
@@ -167,6 +177,8 @@ EXPORTS = {
     "sph_ens_set_search": (C.c_int, [C.c_void_p, C.c_int]),
     "sph_ens_set_blocks": (C.c_int, [C.c_void_p, C.c_uint32, C.c_uint32]),
     "sph_ens_set_graph": (C.c_int, [C.c_void_p, C.c_int]),
+    "sph_ens_set_path": (C.c_int, [C.c_void_p, C.c_int]),
+    "sph_ens_get_path": (C.c_int, [C.c_void_p, C.POINTER(SphPath)]),
     "sph_ens_set_profiling": (C.c_int, [C.c_void_p, C.c_int]),
     "sph_ens_get_timing": (C.c_int, [C.c_void_p, C.POINTER(SphTiming)]),
 }
@@ -376,6 +388,18 @@ class DEM:
             prec = {"fp64": PREC_FP64, "mixed": PREC_MIXED}[prec]
         self._check(self._lib.sph_set_precision(self._h, int(prec)))
 
+    def set_path(self, path: str = "auto"):
+        """How steps run where the kernels are left automatic: "auto",
+        "chain" or "stages" (sph_set_path); the bits are the same."""
+        self._check(self._lib.sph_set_path(self._h, PATHS[path]))
+
+    def path(self) -> Dict[str, int]:
+        """Steps run as a chain and as stages, the chain's launches and its
+        lanes a sphere (sph_get_path)."""
+        out = SphPath()
+        self._check(self._lib.sph_get_path(self._h, C.byref(out)))
+        return {k: int(getattr(out, k)) for k, _ in SphPath._fields_}
+
     def set_profiling(self, on: bool = True):
         self._check(self._lib.sph_set_profiling(self._h, 1 if on else 0))
 
@@ -496,6 +520,18 @@ class Ensemble:
 
     def set_graph(self, on: bool = True):
         self._check(self._lib.sph_ens_set_graph(self._h, 1 if on else 0))
+
+    def set_path(self, path: str = "auto"):
+        """How steps run where the kernels are left automatic: "auto",
+        "chain" or "stages" (sph_ens_set_path); the bits are the same."""
+        self._check(self._lib.sph_ens_set_path(self._h, PATHS[path]))
+
+    def path(self) -> Dict[str, int]:
+        """Steps run as a chain and as stages, the chain's launches and its
+        lanes a sphere (sph_ens_get_path)."""
+        out = SphPath()
+        self._check(self._lib.sph_ens_get_path(self._h, C.byref(out)))
+        return {k: int(getattr(out, k)) for k, _ in SphPath._fields_}
 
     def set_profiling(self, on: bool = True):
         self._check(self._lib.sph_ens_set_profiling(self._h, 1 if on else 0))

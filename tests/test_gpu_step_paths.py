@@ -1,0 +1,121 @@
+"""Both ways through a step, each forced and each shown to have run: a chain of
+like launches and the graph of stages, for systems above the size of four lanes
+a sphere and for ensembles (where timing chooses between them otherwise)."""
+
+import numpy as np
+import pytest
+
+from parity import all_fields, compare_all
+from sphere_amd import configs
+
+pytestmark = pytest.mark.gpu
+
+MEMBER_FIELDS = ["x", "vel", "angvel", "force", "torque", "angpos", "vel0", "angvel0", "xysum", "es_dot", "es", "ev_dot",
+                 "ev", "p", "contacts", "delta_t", "walls_nx", "walls_mvfd", "walls_vel0", "wall_pp", "time"]
+
+
+def _bits(a):
+    return a.view(np.uint64) if a.dtype == np.float64 else a
+
+
+def _ran(dem, path, steps):
+    """The steps counted on the path, and on no other."""
+    p = dem.path()
+    assert (p["chain_steps"], p["stage_steps"]) == ((steps, 0) if path == "chain" else (0, steps)), p
+    assert (p["chain_launches"] >= steps) == (path == "chain")
+    return p["lanes"]
+
+
+def _lattice(nside, seed, moving=0.01, speed=3.0):
+    sb = configs.lattice_settle(nside=nside, spacing=2.0e-2, jitter=2e-5, r_lo=0.998e-2, r_hi=1.002e-2, gamma_n=0.0,
+                                gamma_t=10.0, nw=1)
+    sb.wmode = np.array([1], dtype=np.int32)
+    sb.w_devs[0] = 1e3
+    sb.w_vel[0] = -0.01
+    rng = np.random.default_rng(seed)
+    sb.vel = np.where(rng.random((sb.np, 1)) < moving, rng.uniform(-speed, speed, (sb.np, 3)), 0.0)
+    return sb
+
+
+@pytest.mark.parametrize("path", ["chain", "stages"])
+@pytest.mark.parametrize("nside,lanes", [((20, 21, 22), 4), ((42, 41, 41), 1)])
+def test_one_system_against_the_oracle(nside, lanes, path, tmp_path):
+    from oracle_lib import Oracle
+    from sphere_amd.dem import DEM
+
+    sb = _lattice(nside, 3)
+    dem, orc = DEM(sb, verbosity=0), Oracle.from_spherebin(sb, tmp_path)
+    dem.set_path(path)
+    done = 0
+    for steps in (1, 2, 17):
+        dem.step(steps)
+        done += steps
+        assert orc.step(steps) == 0
+        assert _ran(dem, path, done) == lanes
+        errs = compare_all(dem, orc, all_fields(orc))
+        assert not errs, errs
+    dem.close()
+
+
+@pytest.mark.parametrize("nside", [(20, 21, 22), (42, 41, 41)])
+def test_one_system_in_mixed_precision(nside):
+    """The two paths against each other (the oracle computes in FP64)."""
+    from sphere_amd.dem import DEM
+
+    sb = _lattice(nside, 4)
+    got = []
+    for path in ("chain", "stages"):
+        dem = DEM(sb, verbosity=0)
+        dem.set_precision("mixed")
+        dem.set_path(path)
+        dem.step(1)
+        dem.step(24)
+        _ran(dem, path, 25)
+        got.append({f: dem.get(f) for f in MEMBER_FIELDS})
+        dem.close()
+    for f in MEMBER_FIELDS:
+        assert np.array_equal(_bits(got[0][f]), _bits(got[1][f])), f
+
+
+@pytest.mark.parametrize("path", ["chain", "stages"])
+@pytest.mark.parametrize("sides", [((6, 6, 6), (4, 5, 9), (1, 1, 1)), ((26, 26, 26), (6, 6, 6))])
+def test_ensemble_members_against_their_own_handles(sides, path):
+    """Members with up to 64 wall-sum blocks, whose walls take one launch of the
+    chain, and one with more (17,576 spheres), which takes two."""
+    from sphere_amd.dem import DEM, Ensemble
+
+    sbs = [_lattice(s, 10 + k) if np.prod(s) > 1 else configs.lattice_settle(nside=s, spacing=2.1e-2, jitter=0.0, nw=1, periodic=0)
+           for k, s in enumerate(sides)]
+    ens = Ensemble(sbs)
+    ens.set_path(path)
+    ens.step(1)
+    ens.step(30)
+    assert _ran(ens, path, 31) == 1
+    for k, sb in enumerate(sbs):
+        dem = DEM(sb, verbosity=0)
+        dem.step(1)
+        dem.step(30)
+        for f in MEMBER_FIELDS:
+            assert np.array_equal(_bits(ens.get(k, f)), _bits(dem.get(f))), (k, f)
+        dem.close()
+    ens.close()
+
+
+@pytest.mark.parametrize("sides", [((6, 6, 6), (4, 5, 9)), ((26, 26, 26), (6, 6, 6))])
+def test_ensemble_in_mixed_precision(sides):
+    from sphere_amd.dem import Ensemble
+
+    sbs = [_lattice(s, 20 + k) for k, s in enumerate(sides)]
+    got = []
+    for path in ("chain", "stages"):
+        ens = Ensemble(sbs)
+        ens.set_precision("mixed")
+        ens.set_path(path)
+        ens.step(1)
+        ens.step(30)
+        _ran(ens, path, 31)
+        got.append([{f: ens.get(k, f) for f in MEMBER_FIELDS} for k in range(len(sbs))])
+        ens.close()
+    for a, b in zip(*got):
+        for f in MEMBER_FIELDS:
+            assert np.array_equal(_bits(a[f]), _bits(b[f])), f
