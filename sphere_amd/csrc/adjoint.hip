@@ -658,6 +658,7 @@ struct AdjointState {
     std::vector<Checkpoint> cps;  // one per segment
     Checkpoint end;
     // tape, seg steps
+    bool tape_ready = false;  // all of it and of the adjoint buffers is there
     double4 *tx = nullptr, *tv = nullptr, *tw = nullptr, *twn = nullptr, *twm = nullptr;
     uint32_t *tid = nullptr, *tpos = nullptr, *tmask = nullptr, *tfresh = nullptr, *tslot = nullptr;
     double* tcdt = nullptr;
@@ -679,12 +680,45 @@ void free_adj(AdjointState* a) { delete a; }
 template <class T> int adj_alloc(sph_dem* h, AdjointState* s, T** p, size_t count) {
     void* q = nullptr;
     if (hipMalloc(&q, count * sizeof(T) > 0 ? count * sizeof(T) : 1) != hipSuccess) {
+        (void)hipGetLastError();  // (the next launch's check is not to find it)
         h->err = "adjoint: hipMalloc of " + std::to_string(count * sizeof(T)) + " bytes failed";
         return SPH_E_HIP;
     }
     s->allocs.push_back(q);
     *p = (T*)q;
     return SPH_OK;
+}
+
+// The tape of one segment and the adjoint buffers: all of them, or none (a
+// call that ran out of memory can be made again).
+int alloc_tape(sph_dem* h, AdjointState* a) {
+    const size_t n = h->hs.np, nc = NC, S = a->seg, before = a->allocs.size();
+    auto make = [&]() -> int {
+        int rc;
+        if ((rc = adj_alloc(h, a, &a->tx, S * n)) || (rc = adj_alloc(h, a, &a->tv, S * n)) ||
+            (rc = adj_alloc(h, a, &a->tw, S * n)) || (rc = adj_alloc(h, a, &a->twn, S * 6)) ||
+            (rc = adj_alloc(h, a, &a->twm, S * 6)) || (rc = adj_alloc(h, a, &a->tid, S * n)) ||
+            (rc = adj_alloc(h, a, &a->tpos, S * n)) || (rc = adj_alloc(h, a, &a->tmask, S * n)) ||
+            (rc = adj_alloc(h, a, &a->tfresh, S * n)) || (rc = adj_alloc(h, a, &a->tslot, S * n * nc)) ||
+            (rc = adj_alloc(h, a, &a->gfa, n)) || (rc = adj_alloc(h, a, &a->gfb, n)))
+            return rc;
+        if (a->precision == SPH_PREC_MIXED) rc = adj_alloc(h, a, &a->tcdt32, S * n * nc * 3);
+        else rc = adj_alloc(h, a, &a->tcdt, S * n * nc * 3);
+        if (rc) return rc;
+        for (auto& l : a->lam) {
+            if ((rc = adj_alloc(h, a, &l.x, n)) || (rc = adj_alloc(h, a, &l.v0, n)) || (rc = adj_alloc(h, a, &l.v, n)) ||
+                (rc = adj_alloc(h, a, &l.w0, n)) || (rc = adj_alloc(h, a, &l.w, n)) ||
+                (rc = adj_alloc(h, a, &l.dt, n * nc * 3)) || (rc = adj_alloc(h, a, &l.wall, 3 * 6)))
+                return rc;
+        }
+        return SPH_OK;
+    };
+    const int rc = make();
+    if (rc) {
+        for (size_t k = before; k < a->allocs.size(); ++k) (void)hipFree(a->allocs[k]);
+        a->allocs.resize(before);
+    }
+    return rc;
 }
 
 int read_flags(sph_dem* h) {
@@ -807,24 +841,9 @@ int sph_adjoint_backward(sph_t* h, double grad_out[4]) {
     const size_t n = h->hs.np, nc = sph::NC, S = a->seg;
     int rc;
     // tape and adjoint buffers on first use
-    if (!a->tx) {
-        if ((rc = sph::adj_alloc(h, a, &a->tx, S * n)) || (rc = sph::adj_alloc(h, a, &a->tv, S * n)) ||
-            (rc = sph::adj_alloc(h, a, &a->tw, S * n)) || (rc = sph::adj_alloc(h, a, &a->twn, S * 6)) ||
-            (rc = sph::adj_alloc(h, a, &a->twm, S * 6)) || (rc = sph::adj_alloc(h, a, &a->tid, S * n)) ||
-            (rc = sph::adj_alloc(h, a, &a->tpos, S * n)) || (rc = sph::adj_alloc(h, a, &a->tmask, S * n)) ||
-            (rc = sph::adj_alloc(h, a, &a->tfresh, S * n)) || (rc = sph::adj_alloc(h, a, &a->tslot, S * n * nc)) ||
-            (rc = sph::adj_alloc(h, a, &a->gfa, n)) || (rc = sph::adj_alloc(h, a, &a->gfb, n)))
-            return rc;
-        if (h->precision == SPH_PREC_MIXED) rc = sph::adj_alloc(h, a, &a->tcdt32, S * n * nc * 3);
-        else rc = sph::adj_alloc(h, a, &a->tcdt, S * n * nc * 3);
-        if (rc) return rc;
-        for (auto& l : a->lam) {
-            if ((rc = sph::adj_alloc(h, a, &l.x, n)) || (rc = sph::adj_alloc(h, a, &l.v0, n)) ||
-                (rc = sph::adj_alloc(h, a, &l.v, n)) || (rc = sph::adj_alloc(h, a, &l.w0, n)) ||
-                (rc = sph::adj_alloc(h, a, &l.w, n)) || (rc = sph::adj_alloc(h, a, &l.dt, n * nc * 3)) ||
-                (rc = sph::adj_alloc(h, a, &l.wall, 3 * 6)))
-                return rc;
-        }
+    if (!a->tape_ready) {
+        if ((rc = sph::alloc_tape(h, a))) return rc;
+        a->tape_ready = true;
     }
     hipStream_t st = h->stream;
     auto zero = [&](double* p, size_t count) { sph::k_fill_f64<<<sph::nb(count), 256, 0, st>>>(p, count); };

@@ -35,3 +35,38 @@ def test_recorded_chain_matches_hooks(precision, steps, segment):
         assert a[0] == pytest.approx(b[0], rel=1e-9)
         assert np.allclose(a[1], b[1], rtol=1e-9, atol=0.0)
         assert np.array_equal(a[2], b[2]) and np.array_equal(a[3], b[3])
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_tape_that_does_not_fit_leaves_nothing_half_made(precision):
+    """A segment whose tape is more than the card holds (5.6e8 particle-steps:
+    134 GB, which fit, and then springs of 430 GB or, in FP32, 215 GB): the call
+    is refused each time it is made, and what follows runs as if it had not been
+    made."""
+    from sphere_amd.dem import DEM, HipError
+
+    sb = configs.fcc_shear(cells=(5, 6, 5))
+    w = np.zeros((sb.np, 3))
+    w[np.asarray(sb.vel)[:, 0] > 0.0, 0] = -1.0 / (sb.L[0] * sb.L[1])
+    segment = int(5.6e8 / sb.np)
+    got = []
+    for refused in (True, False):
+        dem = DEM(sb, verbosity=0)
+        dem.set_precision(precision)
+        if refused:
+            dem.adjoint_forward(2, w, segment)
+            for _ in range(2):
+                with pytest.raises(HipError):
+                    dem.adjoint_backward()
+            dem.adjoint_forward(2, w, segment)
+            with pytest.raises(HipError):
+                dem.adjoint_backward()
+        else:
+            dem.step(4)
+        dem.step(1)
+        got.append((dem.adjoint_forward(3, w, 2), dem.adjoint_backward(), dem.get("x"), dem.get("delta_t")))
+        dem.close()
+    a, b = got
+    assert a[0] == pytest.approx(b[0], rel=1e-9)
+    assert np.allclose(a[1], b[1], rtol=1e-9, atol=0.0)
+    assert np.array_equal(a[2], b[2]) and np.array_equal(a[3], b[3])
