@@ -256,7 +256,8 @@ struct DemDev {
                         // (valid with the hint: both are written when the partner is found in a slot)
     uint8_t* nhint;     // mode 5: np * NLIST, the slot where the entry's partner was last found (a hint,
                         // checked against the slot word before use; >= 32 for none), transposed like nlist
-    float* nfree;       // mode 5: per list index, what list_search left (see there); 0: nothing
+    float* nfree;       // mode 5, chains of one lane a sphere: per list index, what list_search left (see there);
+                        // 0: nothing
     const float* ldisp; // mode 5: displacement since the build at the step's start, per list index (FP32)
     float* ldisp_out;   // ... at its end
     float* ldisp2[2];   // the two arrays behind them

@@ -597,6 +597,7 @@ void free_all(sph_dem* h) {
 void sph::enqueue_step(sph_dem* h, bool timed, int parity, bool lead, bool tail, bool outputs, const StepHooks* hooks) {
     DemDev d = step_view(h, parity);
     d.outputs = outputs ? 1u : 0u;
+    h->nfree_stale = true;
     hipStream_t s = h->stream;
     // cell ids and per-cell counts come from the previous step's force
     // kernel (or prepare_keys)
@@ -1112,6 +1113,7 @@ int stage_steps(sph_dem* h, uint64_t n) {
             hipGraphExec_t g = nullptr;
             if ((rc = step_graph(h, lead, h->own_cur, outputs, &g))) return rc;
             HIP_TRY(hipGraphLaunch(g, h->stream));
+            h->nfree_stale = true;
         } else {
             sph::enqueue_step(h, false, h->own_cur, lead, false, outputs);
         }
@@ -1246,6 +1248,10 @@ int sph::chain_steps(sph_dem* h, uint32_t m, const Recording* rec) {
     const DemDev d = sph::step_view(h, h->own_cur);
     int rc;
     if ((rc = upload_views(h, rec))) return rc;
+    if (h->nfree_stale) {
+        sph::launch_fill_u32(reinterpret_cast<uint32_t*>(d.nfree), d.np, 0u, h->stream);
+        h->nfree_stale = false;
+    }
     const DemDev* const views = h->views + h->own_cur * sph::CHAIN_VIEWS;
     // (the launches a step takes follow from how often spheres change cells and
     // lists are due: the last call's mean, and the rest once it is known)

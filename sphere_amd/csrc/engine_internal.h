@@ -32,6 +32,7 @@ struct sph_dem {
     sph::DemDev* views = nullptr;   // step views of a chain, and what they were uploaded from
     std::vector<sph::DemDev> views_host;
     double chain_rate = 1.0;        // launches a step of a chain takes
+    bool nfree_stale = false;       // a step ran as stages, which do not keep DemDev::nfree
     int own_cur = 0;  // 0: the current private records are in b, 1: in a
     bool use_graph = true;
     int precision = SPH_PREC_FP64;

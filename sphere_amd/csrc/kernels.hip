@@ -1720,7 +1720,11 @@ __device__ __forceinline__ uint64_t list_pair(const Sys& S, uint32_t sb, uint32_
 // smallest gap of the entries whose partner holds no slot (negative if one of
 // the slots carries a periodic image; 0 if some gap could close before the
 // lists are built again).  Until a contact of the particle ends, which the
-// force kernel notes there, those gaps stay the only way to a new contact.  A
+// force phase notes there, those gaps stay the only way to a new contact.  (Kept
+// by chains of one lane a sphere alone: stages may give a slot an image without
+// a word of it here, so the first chain after them starts from 0s, and quads
+// neither read nor write it -- a handle's spheres, and with them its lanes a
+// sphere, are the same from open to close.)  A
 // dense packing at rest then reads 4 bytes of search a sphere instead of 13 a
 // list entry and its slot words: crystal of 1,048,576 spheres 424 -> 394 us a
 // step, mixed precision 332 -> 293.  A particle without contacts has a short
@@ -2291,7 +2295,7 @@ __device__ __forceinline__ void finish_particle(const DemDev& d, const Sys& S, W
         raise(wraps, &d.fw[FW_WRAP], 1u);
         const uint32_t li = d.slidx[s];
         d.wo.lidx[s] = li;
-        if (ended) d.nfree[li] = 0.0f;
+        if (CHAIN && ended) d.nfree[li] = 0.0f;
         const float4 xr = d.xref[li];
         float ddx = (float)px - xr.x, ddy = (float)py - xr.y;
         const float ddz = (float)pz - xr.z;

@@ -119,3 +119,54 @@ def test_ensemble_in_mixed_precision(sides):
     for a, b in zip(*got):
         for f in MEMBER_FIELDS:
             assert np.array_equal(_bits(a[f]), _bits(b[f])), f
+
+
+def _pair_about_two_faces():
+    """Two touching spheres a cell apart, both turning round a cell face (one
+    of them the periodic one) within the lists' reach: b to the left of the
+    periodic face in steps 3 to 5 only, a to the right of its own in the steps
+    in which b is not."""
+    from sphere_amd.spherebin import Spherebin
+
+    D, dt = 0.02, 1e-4
+    sb = Spherebin(2, nw=0, sid="two-faces")
+    sb.set_walls(0)
+    configs._contact_params(sb, k_n=1e3, k_t=1e3, gamma_n=0.0, gamma_t=0.0)
+    sb.radius = np.full(2, D / 2)
+    sb.x = np.array([[0.028 * D, 2.5 * D, 2.5 * D], [1.026 * D, 2.5 * D, 2.5 * D]])
+    sb.vel = np.array([[-0.018 * D / dt, 0.0, 0.0]] * 2)
+    configs._grid(sb, [8 * D, 6 * D, 6 * D], 0.999999 * D)
+    assert tuple(sb.num) == (8, 6, 6)
+    sb.periodic = 1
+    sb.g = np.array([0.004 * D / dt ** 2, 0.0, 0.0])
+    sb.time_dt = dt
+    sb.time_total = sb.time_file_dt = 1.0
+    return sb
+
+
+@pytest.mark.parametrize("switch", ["profiling", "graph"])
+def test_stages_between_chain_steps_that_change_an_image(switch):
+    """What a chain's search has noted about a sphere's contacts (that none goes
+    through a periodic face) does not outlast steps taken as stages."""
+    from sphere_amd.dem import Ensemble
+
+    sbs = [_pair_about_two_faces(), _pair_about_two_faces()]
+    got = []
+    for path in ("chain", "stages"):
+        ens = Ensemble(sbs)
+        ens.set_path(path)
+        ens.step(3)
+        ens.set_profiling(switch == "profiling")
+        ens.set_graph(switch != "graph")
+        ens.step(3)
+        ens.set_profiling(False)
+        ens.set_graph(True)
+        ens.step(1)
+        p = ens.path()
+        assert (p["chain_steps"], p["stage_steps"]) == ((4, 3) if path == "chain" else (0, 7)), p
+        got.append([{f: ens.get(k, f) for f in MEMBER_FIELDS if not f.startswith("wall")} for k in range(2)])
+        ens.close()
+    assert np.all(got[1][0]["force"][:, 0] != 0.0)  # the pair touches in the last step
+    for a, b in zip(*got):
+        for f in a:
+            assert np.array_equal(_bits(a[f]), _bits(b[f])), f
