@@ -1244,6 +1244,10 @@ int upload_views(sph_dem* h, const sph::Recording* rec) {
 
 }  // namespace
 
+// Steps of a long call, and steps over which the mean of long calls is taken.
+constexpr uint32_t CHAIN_LONG = 16;
+constexpr double CHAIN_MEMORY = 64.0;
+
 int sph::chain_steps(sph_dem* h, uint32_t m, const Recording* rec) {
     const DemDev d = sph::step_view(h, h->own_cur);
     int rc;
@@ -1254,8 +1258,12 @@ int sph::chain_steps(sph_dem* h, uint32_t m, const Recording* rec) {
     }
     const DemDev* const views = h->views + h->own_cur * sph::CHAIN_VIEWS;
     // (the launches a step takes follow from how often spheres change cells and
-    // lists are due: the last call's mean, and the rest once it is known)
-    uint32_t l = 0, todo = (uint32_t)std::ceil(m * h->chain_rate) + 1, used = 0;
+    // lists are due: the mean of calls before, and the rest once it is known.
+    // Short calls have a mean of their own, the last one's: one that sorts and
+    // builds lists, as the first after sph_set does, takes six launches a step,
+    // and the next long call would be given as many)
+    double& mean = h->chain_rate[m >= CHAIN_LONG ? 1 : 0];
+    uint32_t l = 0, todo = (uint32_t)std::ceil(m * mean) + 1, used = 0;
     for (;;) {
         for (uint32_t k = 0; k < todo; ++k) sph::launch_chain(d, views, h->precision, m, l++, h->stream);
         HIP_TRY(hipGetLastError());
@@ -1267,7 +1275,7 @@ int sph::chain_steps(sph_dem* h, uint32_t m, const Recording* rec) {
         const double rate = steps ? (double)used / steps : 5.0;
         todo = (uint32_t)std::ceil((m - steps) * rate) + 1;
     }
-    h->chain_rate = (double)used / m;
+    mean += ((double)used / m - mean) * (m < CHAIN_LONG ? 1.0 : std::min(1.0, m / CHAIN_MEMORY));
     if (m & 1) h->own_cur ^= 1;
     for (uint32_t k = 0; k < m; ++k) h->hs.t_cur += h->hs.dt;
     h->steps_done += m;

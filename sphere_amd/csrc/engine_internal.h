@@ -31,7 +31,7 @@ struct sph_dem {
     uint32_t* control = nullptr;    // pinned: the control words and error flags as last read; get_host behind them
     sph::DemDev* views = nullptr;   // step views of a chain, and what they were uploaded from
     std::vector<sph::DemDev> views_host;
-    double chain_rate = 1.0;        // launches a step of a chain takes
+    double chain_rate[2] = {1.0, 1.0};  // launches a step of a chain takes, in short calls and in long ones
     bool nfree_stale = false;       // a step ran as stages, which do not keep DemDev::nfree
     int own_cur = 0;  // 0: the current private records are in b, 1: in a
     bool use_graph = true;

@@ -170,3 +170,19 @@ def test_stages_between_chain_steps_that_change_an_image(switch):
     for a, b in zip(*got):
         for f in a:
             assert np.array_equal(_bits(a[f]), _bits(b[f])), f
+
+
+def test_launches_of_a_long_call_after_a_short_one():
+    """One step after new positions sorts and builds lists (six launches); the
+    quiet steps of the next call are one launch each."""
+    from sphere_amd.dem import DEM
+
+    sb = configs.lattice_settle(nside=(10, 10, 10), spacing=2.1e-2, jitter=0.0, r_lo=1e-2, r_hi=1e-2, gravity=0.0)
+    dem = DEM(sb, verbosity=0)
+    for _ in range(2):
+        dem.set("x", dem.get("x"))
+        dem.step(1)
+        before = dem.path()["chain_launches"]
+        dem.step(300)
+        assert dem.path()["chain_launches"] - before <= 310
+    dem.close()
