@@ -1233,7 +1233,7 @@ int upload_views(sph_dem* h, const sph::Recording* rec) {
     if (!h->views) {
         int rc;
         if ((rc = dalloc(h, &h->views, v.size()))) return rc;
-    } else if (std::memcmp(v.data(), h->views_host.data(), bytes) == 0) {
+    } else if (h->views_host.size() == v.size() && std::memcmp(v.data(), h->views_host.data(), bytes) == 0) {
         return SPH_OK;
     }
     HIP_TRY(hipMemcpyAsync(h->views, v.data(), bytes, hipMemcpyHostToDevice, h->stream));
@@ -1269,8 +1269,13 @@ int sph::chain_steps(sph_dem* h, uint32_t m, const Recording* rec) {
         HIP_TRY(hipGetLastError());
         if ((rc = read_control(h))) return rc;
         const uint32_t* now = h->control + (l & 1u) * sph::CHAIN_WORDS;
+        const uint32_t before = used;
         used = now[sph::CHAIN_USED] & ~sph::CHAIN_SORTED;
         if (now[sph::CHAIN_PHASE] == sph::PH_TAIL || now[sph::CHAIN_PHASE] == sph::PH_DONE) break;
+        if (used == before) {  // (every launch short of the tail has work and counts)
+            h->err = "a chain of launches came to a stop";
+            return SPH_E_HIP;
+        }
         const uint32_t steps = now[sph::CHAIN_STEPS];
         const double rate = steps ? (double)used / steps : 5.0;
         todo = (uint32_t)std::ceil((m - steps) * rate) + 1;
