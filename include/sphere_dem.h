@@ -370,10 +370,11 @@ int sph_ens_info(const sph_ens_t* e, sph_ens_info_t* out);
 
 /* Kernel choices, as for one handle: precision; search mode 0 (automatic: on
  * the next sph_ens_step the autotuner times the row, half-shell and list
- * kernels and then 64, 128 and 256 threads per block for the search and
- * force kernels, on ordinary steps, and keeps the fastest), 2, 4 or 5 (1 and
- * 3 walk one grid and are refused); graph capture; how steps run
- * (sph_set_path); per-kernel profiling. */
+ * kernels, then 64, 128 and 256 threads per block for the search and force
+ * kernels, then list search and forces as one kernel, on a copy of the state,
+ * and keeps the fastest), 2, 4 or 5 (1 and 3 walk one grid and are refused);
+ * threads per block of the search and force kernels, which then run as stages;
+ * graph capture; how steps run (sph_set_path); per-kernel profiling. */
 int sph_ens_set_precision(sph_ens_t* e, int precision);
 int sph_ens_set_search(sph_ens_t* e, int mode);
 int sph_ens_set_blocks(sph_ens_t* e, uint32_t force_block, uint32_t search_block);

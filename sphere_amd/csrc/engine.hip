@@ -1079,9 +1079,10 @@ int sph::restore_state(sph_dem* h, const Checkpoint& c) {
 // Steps between two readings of the error flags.
 constexpr uint64_t STEP_CHUNK = 512;
 
-// A handle whose kernels the caller left to it, and that may step as a chain.
+// A handle whose kernels the caller left to it (an ensemble's block sizes too),
+// and that may step as a chain.
 static bool automatic(const sph_dem* h) {
-    return h->path != SPH_PATH_STAGES && h->force_auto && (h->search_auto || (h->members.empty() && h->hs.contactmodel == 1));
+    return h->path != SPH_PATH_STAGES && h->force_auto && (h->members.empty() || h->blocks_auto) && (h->search_auto || (h->members.empty() && h->hs.contactmodel == 1));
 }
 
 // ... whose steps are a chain of launches whatever a timing would say: small

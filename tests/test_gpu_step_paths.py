@@ -186,3 +186,26 @@ def test_launches_of_a_long_call_after_a_short_one():
         dem.step(300)
         assert dem.path()["chain_launches"] - before <= 310
     dem.close()
+
+
+def test_block_sizes_of_an_ensemble_are_the_callers():
+    """Set sizes are those of the kernels that run: not of a chain, which has
+    its own."""
+    from sphere_amd.dem import Ensemble
+
+    sbs = [_lattice((6, 6, 6), 1), _lattice((7, 5, 6), 2)]
+    got = []
+    for blocks in (None, (64, 128)):
+        ens = Ensemble(sbs)
+        ens.set_path("chain")
+        if blocks:
+            ens.set_blocks(*blocks)
+        ens.step(10)
+        i = ens.info()
+        if blocks:
+            assert (i.force_block, i.search_block) == blocks
+        _ran(ens, "stages" if blocks else "chain", 10)
+        got.append([ens.get(k, "x") for k in range(2)])
+        ens.close()
+    for a, b in zip(*got):
+        assert np.array_equal(_bits(a), _bits(b))
