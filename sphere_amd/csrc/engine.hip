@@ -1082,7 +1082,7 @@ constexpr uint64_t STEP_CHUNK = 512;
 // A handle whose kernels the caller left to it (an ensemble's block sizes too),
 // and that may step as a chain.
 static bool automatic(const sph_dem* h) {
-    return h->path != SPH_PATH_STAGES && h->force_auto && (h->members.empty() || h->blocks_auto) && (h->search_auto || (h->members.empty() && h->hs.contactmodel == 1));
+    return h->use_graph && h->path != SPH_PATH_STAGES && h->force_auto && (h->members.empty() || h->blocks_auto) && (h->search_auto || (h->members.empty() && h->hs.contactmodel == 1));
 }
 
 // ... whose steps are a chain of launches whatever a timing would say: small
@@ -1178,13 +1178,9 @@ int tune_chain(sph_dem* h) {
 
 int sph::autotune(sph_dem* h) {
     if (chain_only(h)) {  // nothing to choose: neighbour lists (models with slots)
-        if (!h->tuned) {
-            h->tuned = true;
-            h->d.force_vw = 0;
-            if (h->search_auto) {
-                h->d.search_mode = 5;
-                request_list_rebuild(h);
-            }
+        if (h->search_auto && h->d.search_mode != 5) {  // (timing as plain launches may have found another)
+            h->d.search_mode = 5;
+            request_list_rebuild(h);
             destroy_graph(h);
         }
         return SPH_OK;
@@ -1198,7 +1194,7 @@ int sph::autotune(sph_dem* h) {
     // them) is the trial's, not the caller's: the kernels chosen so far are
     // kept and the restored state is stepped as asked
     rc = tune_search(h);
-    if (!rc && automatic(h) && h->use_graph && h->d.search_mode == 5) rc = tune_chain(h);
+    if (!rc && automatic(h) && h->d.search_mode == 5) rc = tune_chain(h);
     if (rc == SPH_E_HIP) return rc;
     h->tuned = true;
     h->steps_since_tune = 0;
@@ -1323,7 +1319,7 @@ int run_steps(sph_dem* h, uint64_t n) {
     }
     if ((rc = sph::autotune(h))) return rc;
     h->steps_since_tune += n;
-    return sph::chained(h) && h->use_graph ? chained_steps(h, n) : stage_steps(h, n);
+    return sph::chained(h) ? chained_steps(h, n) : stage_steps(h, n);
 }
 
 bool field_is_known(int f) { return f >= 0 && f < SPH_NFIELDS; }

@@ -70,3 +70,30 @@ def test_tape_that_does_not_fit_leaves_nothing_half_made(precision):
     assert a[0] == pytest.approx(b[0], rel=1e-9)
     assert np.allclose(a[1], b[1], rtol=1e-9, atol=0.0)
     assert np.array_equal(a[2], b[2]) and np.array_equal(a[3], b[3])
+
+
+def test_plain_launches_are_plain_in_the_adjoint_too():
+    """set_graph(False) asks for one kernel per stage; back on, the same handle
+    steps as a chain again."""
+    from sphere_amd.dem import DEM
+
+    sb = configs.fcc_shear(cells=(5, 6, 5))
+    w = np.zeros((sb.np, 3))
+    w[np.asarray(sb.vel)[:, 0] > 0.0, 0] = -1.0 / (sb.L[0] * sb.L[1])
+    got = []
+    for graph in (True, False):
+        dem = DEM(sb, verbosity=0)
+        dem.set_graph(graph)
+        dem.step(3)
+        got.append((dem.adjoint_forward(7, w, 3), dem.adjoint_backward(), dem.get("x"), dem.get("delta_t")))
+        p = dem.path()
+        assert (p["chain_steps"] > 0, p["stage_steps"] > 0) == (graph, not graph), p
+        dem.set_graph(True)
+        dem.step(5)
+        q = dem.path()
+        assert q["chain_steps"] == p["chain_steps"] + 5 and q["stage_steps"] == p["stage_steps"], q
+        dem.close()
+    a, b = got
+    assert a[0] == pytest.approx(b[0], rel=1e-9)
+    assert np.allclose(a[1], b[1], rtol=1e-9, atol=0.0)
+    assert np.array_equal(a[2], b[2]) and np.array_equal(a[3], b[3])
