@@ -209,3 +209,56 @@ def test_block_sizes_of_an_ensemble_are_the_callers():
         ens.close()
     for a, b in zip(*got):
         assert np.array_equal(_bits(a), _bits(b))
+
+
+def _large_among_small(side=17, ratio=6.0):
+    """A sphere with more small neighbours within the lists' reach than a list
+    holds (48), none of them touching it."""
+    from sphere_amd.spherebin import Spherebin
+
+    r, a = 1e-3, 2.2e-3
+    L = np.full(3, side * a)
+    x = (np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing="ij"), -1).reshape(-1, 3) + 0.5) * a
+    R = ratio * r
+    x = x[np.linalg.norm(x - L / 2, axis=1) > R + 1.01 * r]
+    sb = Spherebin(len(x) + 1, nw=0, sid="large-among-small")
+    sb.set_walls(0)
+    configs._contact_params(sb, gamma_n=0.0, gamma_t=10.0)
+    sb.x = np.concatenate([x, [L / 2]])
+    sb.radius = np.concatenate([np.full(len(x), r), [R]])
+    configs._grid(sb, L, 2 * R)
+    sb.periodic = 1
+    sb.g = np.zeros(3)
+    sb.time_dt = configs._dt(sb)
+    sb.time_total = sb.time_file_dt = 1.0
+    sb.vel = np.random.default_rng(1).uniform(-0.5, 0.5, (sb.np, 3))
+    return sb
+
+
+@pytest.mark.parametrize("path", ["chain", "stages"])
+def test_neighbour_list_that_overflows(path, tmp_path):
+    """Such a list is no use and is built at every step; four lanes a sphere
+    against the oracle, one lane (an ensemble) against those."""
+    from oracle_lib import Oracle
+    from sphere_amd.dem import DEM, Ensemble
+
+    sb = _large_among_small()
+    near = np.linalg.norm(sb.x[:-1] - sb.x[-1], axis=1) < sb.radius[0] + sb.radius[-1] + 0.1 * np.min(sb.L / sb.num)
+    assert near.sum() > 48
+    dem, orc, ens = DEM(sb, verbosity=0), Oracle.from_spherebin(sb, tmp_path), Ensemble([sb, sb])
+    dem.set_path(path)
+    ens.set_path(path)
+    for steps in (1, 9, 30):
+        dem.step(steps)
+        ens.step(steps)
+        assert orc.step(steps) == 0
+        errs = compare_all(dem, orc, all_fields(orc))
+        assert not errs, errs
+    if path == "chain":
+        assert dem.timing()["list_builds"] == ens.timing()["list_builds"] == 40
+        assert _ran(dem, path, 40) == 4 and _ran(ens, path, 40) == 1
+    for f in MEMBER_FIELDS:
+        if not f.startswith("wall"):
+            assert np.array_equal(_bits(ens.get(1, f)), _bits(dem.get(f))), f
+    dem.close()
+    ens.close()
