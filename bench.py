@@ -18,8 +18,10 @@ bonds) over 5,000 steps; and the 512-member calibration ensemble stepped in
 one handle against the same members one at a time; and the reference's
 analysis members (porosity, pair overlaps) on the dense crystal.  Per-kernel time comes
 from hipEvents recorded on the simulation's own stream around each stage,
-over a separate run of the same steps; the roofline entry is for the stage
-with the largest share of the step.
+over a separate run of the same steps as stages.  Where the timed steps ran as
+a chain of launches (one kernel for search, forces and the rest of a step) the
+roofline entry is for that kernel over the whole timed step, otherwise for the
+stage with the largest share.
 """
 
 from __future__ import annotations
@@ -53,6 +55,43 @@ SEARCH_KERNELS = {1: "k_topo", 2: "k_topo_rows", 3: "k_topo_wave", 4: "k_topo_ha
                   5: "k_list_search (k_topo_rows<true> on rebuild steps)"}
 SEARCH_PROFILE = {1: "k_topo", 2: "k_topo_rows<false, false>", 3: "k_topo_wave", 4: "k_topo_half<false>",
                   5: "k_list_search<false>"}
+
+
+# what runs when steps are a chain (one lane a sphere, contact model 2)
+CHAIN_KERNELS = {("fp64", False): "k_chain<double, 2, false, false>", ("mixed", False): "k_chain<float, 2, false, false>",
+                 ("fp64", True): "k_chain<double, 2, false, true>", ("mixed", True): "k_chain<float, 2, false, true>"}
+STAGES_NOTE = "per-stage times of a separate run of the same steps as stages"
+
+
+def timed_as(before, after):
+    """How the steps between two readings of path() ran."""
+    chain, stages = (after[k] - before[k] for k in ("chain_steps", "stage_steps"))
+    if chain and stages:
+        return {"as": "chain and stages", "launches_per_step": None}
+    return {"as": "chain" if chain else "stages",
+            "launches_per_step": (after["chain_launches"] - before["chain_launches"]) / chain if chain else None}
+
+
+def search_label(timed, precision, search_mode, ensemble=False):
+    """The kernel that searched for contacts in the timed steps."""
+    if timed["as"] == "chain":
+        return "neighbour lists, in " + CHAIN_KERNELS[precision, ensemble]
+    return SEARCH_KERNELS.get(search_mode, "?")
+
+
+def step_roofline_entry(timed, precision, kb, ms, stage_ms, stage_kernels, profile_kernel, summary):
+    """Roofline of the kernel that took the timed steps: as a chain, k_chain
+    with the force, wall and bond bytes of a step over the step's time (a step
+    that sorts moves more, and one whose lists are read; those are left out);
+    as stages, the stage with the largest share, by its own events."""
+    if timed["as"] == "chain":
+        name = CHAIN_KERNELS[precision, False]
+        e = roofline_entry(name, kb["force"] + kb["walls"] + kb["bonds"], ms,
+                           measured_traffic(name + " force phase", summary))
+        return dict(e, timed="whole steps, all launches", launches_per_step=timed["launches_per_step"])
+    dom = max(stage_ms, key=lambda k: stage_ms[k])
+    e = roofline_entry(stage_kernels[dom], kb[dom], stage_ms[dom], measured_traffic(profile_kernel.get(dom), summary))
+    return dict(e, timed=STAGES_NOTE)
 
 
 def log(msg):
@@ -138,9 +177,11 @@ def timed_run(bin_path, precision, steps, warmup, prof_steps):
     dem.step(warmup)
     # sph_step returns after the device finished the steps (it reads back the
     # error flags), so the timed region is bracketed by device syncs
+    ran = dem.path()
     t0 = time.perf_counter()
     dem.step(steps)
     ms = (time.perf_counter() - t0) * 1e3 / steps
+    timed = timed_as(ran, dem.path())
     c = int((dem.get("contacts") != n).sum())
     dem.set_profiling(True)
     dem.step(prof_steps)
@@ -151,7 +192,7 @@ def timed_run(bin_path, precision, steps, warmup, prof_steps):
              "wall_pp0": dem.get("wall_pp")[0].copy() if info.nw else None}
     dem.close()
     stage_ms = {k: tim[f"{k}_ms"] / max(1, tim["steps"]) for k in STAGES}
-    return {"ms": ms, "contacts": c, "stage_ms": stage_ms, "tile": [tim["tile_x"], tim["tile_y"]],
+    return {"ms": ms, "timed": timed, "contacts": c, "stage_ms": stage_ms, "tile": [tim["tile_x"], tim["tile_y"]],
             "search_mode": int(tim["search_mode"]), "force_variant": int(tim["force_variant"]), "state": state,
             "steps_total": warmup + steps + prof_steps}
 
@@ -226,9 +267,11 @@ def bonded_run(tmp, steps, warmup, prof_steps):
     n, nb = sb.np, sb.nb0
     dem = DEM(path, verbosity=0)
     dem.step(warmup)
+    ran = dem.path()
     t0 = time.perf_counter()
     dem.step(steps)
     ms = (time.perf_counter() - t0) * 1e3 / steps
+    timed = timed_as(ran, dem.path())
     broken = int((dem.get("bonds")[:, 0] >= n).sum())
     dem.set_profiling(True)
     dem.step(prof_steps)
@@ -240,7 +283,8 @@ def bonded_run(tmp, steps, warmup, prof_steps):
     return {"workload": f"{n:,}-sphere jittered FCC solid, {nb:,} bonds (d <= 1.05 (r_i + r_j)), k = 1e7, "
                         f"sigma_b = tau_b = 1e5 Pa, top and bottom layers pulled apart at 0.01 m/s, FP64",
             "n": n, "bonds": nb, "steps": steps, "warmup": warmup, "value": n / (ms * 1e-3),
-            "unit": "particle-steps/s", "ms_per_step": ms, "broken_bonds": broken, "stage_ms": stage_ms,
+            "unit": "particle-steps/s", "ms_per_step": ms, "timed": timed, "broken_bonds": broken, "stage_ms": stage_ms,
+            "stage_ms_note": STAGES_NOTE,
             "k_bonds": {"algorithmic_bytes": bonds_bytes, "GBs": bonds_bytes / (stage_ms["bonds"] * 1e-3) / 1e9
                         if stage_ms["bonds"] > 0 else None}}
 
@@ -334,9 +378,8 @@ def regrid(sb, factor):
 
 
 def ensemble_run(members, steps, warmup, sample_every=1, sample_steps=None):
-    """The calibration ensemble in one handle (one launch of each kernel per
-    step for every member, graph-replayed), mixed precision, grid and block
-    sizes from the autotuner; against the same members run one at a time,
+    """The calibration ensemble in one handle (a step's launches serve every
+    member), mixed precision, grid and kernels from the autotuner; against the same members run one at a time,
     each in its own handle for the same steps (every member by default;
     `sample_every` > 1 extrapolates a sample by member count)."""
     sample_steps = sample_steps or steps
@@ -348,9 +391,11 @@ def ensemble_run(members, steps, warmup, sample_every=1, sample_steps=None):
     t_open = time.perf_counter() - t0
     ens.set_precision("mixed")
     ens.step(warmup)  # the first call also tunes the search kernel and the block sizes (on a copy)
+    ran = ens.path()
     t0 = time.perf_counter()
     ens.step(steps)
     ms = (time.perf_counter() - t0) * 1e3 / steps
+    timed = timed_as(ran, ens.path())
     info = ens.info()
     ens.set_profiling(True)
     ens.step(20)
@@ -376,9 +421,10 @@ def ensemble_run(members, steps, warmup, sample_every=1, sample_steps=None):
                         "in [1e5, 1e7], mu uniform in [0.2, 0.8], C1 radii, settling under a 10 kPa top wall, mixed "
                         "precision",
             "members": len(members), "n": n_total, "steps": steps, "warmup": warmup,
-            "value": n_total / (ms * 1e-3), "unit": "particle-steps/s", "ms_per_step": ms, "stage_ms": stage_ms,
+            "value": n_total / (ms * 1e-3), "unit": "particle-steps/s", "ms_per_step": ms, "timed": timed,
+            "stage_ms": stage_ms, "stage_ms_note": STAGES_NOTE,
             "autotuned": {"cell_factor": info.cell_factor, "trial_ms_per_step": list(info.tuned_ms),
-                          "search_kernel": SEARCH_KERNELS.get(info.search_mode),
+                          "search_kernel": search_label(timed, "mixed", info.search_mode, True),
                           "force_block": info.force_block, "search_block": info.search_block},
             "one_at_a_time": {"value": n_total / (ms_one * 1e-3), "ms_per_ensemble_step": ms_one,
                               "ms_per_member_step": float(np.mean(per)), "members_timed": len(sample),
@@ -450,7 +496,7 @@ def main():
         sbd.writebin(dpath)
         run = timed_run(dpath, args.profile_dense, args.steps, args.warmup, prof_steps)
         print(json.dumps({"workload": "dense crystal", "n": sbd.np, "precision": args.profile_dense,
-                          "ms_per_step": run["ms"], "contacts_per_particle": run["contacts"] / sbd.np,
+                          "ms_per_step": run["ms"], "timed": run["timed"], "contacts_per_particle": run["contacts"] / sbd.np,
                           "stage_ms": run["stage_ms"], "search_mode": run["search_mode"],
                           "force_variant": run["force_variant"]}), flush=True)
         return
@@ -474,8 +520,6 @@ def main():
     per_kernel = {k: {"ms": stage_ms[k], "kernels": stage_kernels[k], "algorithmic_bytes": kb[k],
                       "GBs": (kb[k] / (stage_ms[k] * 1e-3) / 1e9) if stage_ms[k] > 0 and kb[k] else None}
                   for k in STAGES}
-    dom = max(stage_ms, key=lambda k: stage_ms[k])
-    achieved = kb[dom] / (stage_ms[dom] * 1e-3) / 1e9
     step_b = sum(kb.values())
     result = {
         "metric": METRIC,
@@ -492,13 +536,14 @@ def main():
         "data": "synthetic (seeded lognormal random packing)",
         "config": {"workload": "1,048,576 lognormal spheres, random packing, 10 kPa top wall, 2.07x2.07x4.13 m x/y-periodic box",
                    "n": n, "cells": K, "contacts_per_particle": c / n, "precision": args.precision,
-                   "search_kernel": stage_kernels["search"], "search_mode": main_run["search_mode"]},
+                   "search_kernel": search_label(main_run["timed"], args.precision, main_run["search_mode"]),
+                   "search_mode": main_run["search_mode"], "timed": main_run["timed"]},
         "per_kernel": per_kernel,
-        "roofline": {"bound": "hbm", "kernel": stage_kernels[dom], "achieved": achieved, "peak": HBM_PEAK_GBS,
-                     "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
-                     "traffic": measured_traffic(profile_kernel.get(dom)),
-                     "algorithmic_bytes_per_launch": kb[dom]},
-        "step_roofline": {"algorithmic_bytes": step_b, "achieved_GBs": step_b / (ms * 1e-3) / 1e9,
+        "per_kernel_note": STAGES_NOTE,
+        "roofline": step_roofline_entry(main_run["timed"], args.precision, kb, ms, stage_ms, stage_kernels,
+                                        profile_kernel, "c1_1M_pmc_traffic.md"),
+        "step_roofline": {"note": "a sort and a reorder counted for every step, also for those that make none",
+                          "algorithmic_bytes": step_b, "achieved_GBs": step_b / (ms * 1e-3) / 1e9,
                           "frac": step_b / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS},
     }
     if not args.no_mixed and args.precision == "fp64":
@@ -516,11 +561,15 @@ def main():
         dense = {"workload": "1,048,576-sphere FCC crystal (4 x 64^3), nearest neighbours overlapping by 2e-5 m, "
                              "x/y periodic, floor and fixed top wall, gamma_n = 0",
                  "contacts_per_particle": d64["contacts"] / dn, "fp64": {"value": dn / (d64["ms"] * 1e-3),
-                 "ms_per_step": d64["ms"], "stage_ms": d64["stage_ms"],
-                 "search_kernel": SEARCH_KERNELS.get(d64["search_mode"])}}
+                 "ms_per_step": d64["ms"], "timed": d64["timed"], "stage_ms": d64["stage_ms"],
+                 "stage_ms_note": STAGES_NOTE,
+                 "search_kernel": search_label(d64["timed"], "fp64", d64["search_mode"])}}
         kd = kernel_bytes(dn, d64["contacts"], 0, sbd.nw, int(np.prod(sbd.num.astype(np.int64))))
         dsk = SEARCH_PROFILE.get(d64["search_mode"])
         dense["fp64"]["roofline"] = {
+            "step": step_roofline_entry(d64["timed"], "fp64", kd, d64["ms"], d64["stage_ms"], STAGE_KERNELS,
+                                        dict(PROFILE_KERNEL, search=dsk), "dense_1M_fp64_pmc_traffic.md"),
+            "note": "force and search: " + STAGES_NOTE,
             "force": roofline_entry(FORCE_PROFILE[d64["force_variant"]], kd["force"], d64["stage_ms"]["force"],
                                     measured_traffic(FORCE_PROFILE[d64["force_variant"]], "dense_1M_fp64_pmc_traffic.md")),
             "search": roofline_entry(dsk, kd["search"], d64["stage_ms"]["search"],
@@ -530,7 +579,7 @@ def main():
         if not args.no_mixed:
             dmx = timed_run(dpath, "mixed", args.steps, args.warmup, prof_steps)
             log(f"dense mixed: {dmx['ms']:.4f} ms/step")
-            dense["mixed"] = {"value": dn / (dmx["ms"] * 1e-3), "ms_per_step": dmx["ms"],
+            dense["mixed"] = {"value": dn / (dmx["ms"] * 1e-3), "ms_per_step": dmx["ms"], "timed": dmx["timed"],
                               "speedup_vs_fp64": d64["ms"] / dmx["ms"], "stage_ms": dmx["stage_ms"],
                               "error_vs_fp64": mixed_error(d64, dmx, float(sbd.L[0] * sbd.L[1]),
                                                            float(sbd.radius.min()))}
