@@ -1037,22 +1037,27 @@ int copy_regions(sph_dem* h, const std::vector<Region>& from, const std::vector<
 }  // namespace
 
 sph::Checkpoint::~Checkpoint() {
-    for (void* p : bufs) (void)hipFree(p);
+    (void)hipFree(block);
 }
 
 int sph::save_state(sph_dem* h, Checkpoint& c) {
     const auto regs = state_regions(h, h->own_cur);
     if (c.bufs.size() != regs.size()) {
-        for (void* p : c.bufs) (void)hipFree(p);
+        (void)hipFree(c.block);
+        c.block = nullptr;
         c.bufs.clear();
+        std::vector<size_t> at;
+        size_t bytes = 0;
         for (const Region& r : regs) {
-            void* q = nullptr;
-            if (hipMalloc(&q, r.bytes) != hipSuccess) {
-                h->err = "state copy: hipMalloc of " + std::to_string(r.bytes) + " bytes failed";
-                return SPH_E_HIP;
-            }
-            c.bufs.push_back(q);
+            at.push_back(bytes);
+            bytes += (r.bytes + 255) / 256 * 256;
         }
+        if (hipMalloc(&c.block, bytes) != hipSuccess) {
+            c.block = nullptr;
+            h->err = "state copy: hipMalloc of " + std::to_string(bytes) + " bytes failed";
+            return SPH_E_HIP;
+        }
+        for (size_t a : at) c.bufs.push_back(static_cast<char*>(c.block) + a);
     }
     std::vector<Region> to;
     for (size_t k = 0; k < regs.size(); ++k) to.push_back({c.bufs[k], regs[k].bytes});
@@ -1159,27 +1164,33 @@ int chained_steps(sph_dem* h, uint64_t n) {
 }
 
 // Chain or graph, for lists in a system too large for four lanes a sphere or
-// an ensemble, by the time of eight steps each after eight others.  The chain
-// wins where search and force are most of a step, the graph where most steps
-// sort: each stage then runs at its own occupancy.  us a step as chain and as
-// graph: crystal of 1,048,576 spheres 395 and 463, loose packing of 131,071 35
-// and 53, of 400,000 88 and 97, lattice of 1,000,000 204 and 200, sheared
-// 2,000,000 1,001 and 996, 512 calibration systems of 8,464,166 spheres 1,930
-// and 1,610.
+// an ensemble, by the time of five steps each after three or four others.  The
+// chain wins where search and force are most of a step, the graph where most
+// steps sort or bonds are most of it: each stage then runs at its own
+// occupancy.  us a step as chain and as graph: crystal of 256,000 spheres 110
+// and 139, of 1,048,576 395 and 462; loose packing of 131,071 36 and 56, of
+// 300,000 61 and 80; lattice of 1,000,000 204 and 225; sheared 256,000 132 and
+// 160, 2,000,000 1,001 and 996; bonded 256,000 389 and 311; 64 calibration
+// systems of 112,000 spheres 75 and 77, 512 of 8,464,166 1,930 and 1,610.
+// (The first step of a handle pays for it: crystal of 256,000 9.8 ms with it,
+// where 12.4 were taken by the trials of the stages alone while the copy of the
+// state was thirty-odd allocations.)
 int tune_chain(sph_dem* h) {
     double ms[2];
     for (int chain = 0; chain < 2; ++chain) {
         request_list_rebuild(h);
-        for (int part = 0; part < 3; ++part) {
+        // (the steps before make the lists and the graphs, or show how many
+        // launches a step without new lists takes)
+        for (int part = chain ? 0 : 1; part < 3; ++part) {
             const auto t0 = std::chrono::steady_clock::now();
-            const int rc = chain ? chained_steps(h, part == 2 ? 8 : 4) : stage_steps(h, part == 2 ? 8 : 4);
+            const int rc = chain ? chained_steps(h, part == 2 ? 5 : 2) : stage_steps(h, part == 2 ? 5 : 3);
             if (rc) return rc;
             ms[chain] = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
         }
     }
     h->as_chain = ms[1] < ms[0];
     if (h->verbosity > 1)
-        std::printf("sphere_dem: 8 steps as graph %.4f ms, as chain %.4f ms\n", ms[0], ms[1]);
+        std::printf("sphere_dem: 5 steps as graph %.4f ms, as chain %.4f ms\n", ms[0], ms[1]);
     return SPH_OK;
 }
 
