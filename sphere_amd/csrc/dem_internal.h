@@ -39,10 +39,15 @@ constexpr int BLOCK = 256;
 // Spheres of a system whose chain takes four lanes a sphere, at most: up to
 // here one lane a sphere leaves the chip short of wavefronts (65,536 spheres
 // are one a SIMD), from here on four only add instructions.  us a step with
-// four and with one: crystal of 16,384 spheres 16 and 31, of 62,500 37 and 37,
-// of 131,072 69 and 50; loose packing of 20,000 12 and 15, of 65,000 23 and 20,
-// of 131,071 41 and 26; lattice of 64,000 25 and 24; bonded 62,500 75 and 85,
-// 131,072 143 and 134; sheared 65,536 66 and 74, 128,000 91 and 72.
+// four and with one: bonded 32,000 48 and 77, 62,500 74 and 85, 131,072 143
+// and 134; sheared 16,000 27 and 52, 35,152 45 and 59, 65,536 66 and 74, 128,000
+// 91 and 72; crystal of 16,384 spheres 16 and 27, of 32,000 23 and 32, of
+// 62,500 38 and 34, of 131,072 70 and 46 (mixed precision 14 and 24, 20 and 28,
+// 31 and 31, 52 and 38); lattice of 32,768 14 and 24, of 64,000 26 and 25; loose
+// packing under a moving wall of 20,000 19 and 22, of 40,000 26 and 24, of 65,000
+// 31 and 28, of 100,000 44 and 33.  So the crossing lies between 35,000 (loose)
+// and 100,000 (bonded), and this is a line for all: the widest loss is 12 %, of
+// crystals at 62,500.
 constexpr uint32_t QUAD_NP = 65536;
 // Wall-sum blocks of a system that one workgroup sums on its way to the wall's
 // update; with more the sums take a launch of all workgroups first.  us a step

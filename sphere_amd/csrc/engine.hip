@@ -1101,7 +1101,15 @@ static bool automatic(const sph_dem* h) {
 
 // ... whose steps are a chain of launches whatever a timing would say: small
 // enough for four lanes a sphere, or without a contact search to choose, or at
-// the caller's wish.
+// the caller's wish.  Where the lists serve more than one step nothing else
+// comes near it at these sizes (990 spheres 16 us a step against 47).  Where
+// they are due at every step it is no better than the stages or, with many
+// candidates, worse; us a step as chain, as stages and with the twelve kernels
+// and the search by timing that it replaced: cells no wider than a pair on a
+// periodic axis of four, 4,000 spheres 72, 73 and 108, 60,000 91, 79 and 113; a
+// gas that rebuilds every other step, 59,319 spheres 125, 94 and 144; lists that
+// overflow (radii 5:1), 14,961 spheres 735, 281 and 2,158, 53,863 988, 255 and
+// 2,057.
 static bool chain_only(const sph_dem* h) {
     return automatic(h) && (h->path == SPH_PATH_CHAIN ||
                             (h->members.empty() && (h->hs.np <= sph::QUAD_NP || h->hs.contactmodel == 1)));
@@ -2163,7 +2171,8 @@ int ens_open(std::vector<HostState> ms, int verbosity, sph_ens** out, std::strin
 }
 
 // ms per step of an ensemble on `ms` regridded by `factor`: the autotuner's
-// steps (search kernel and block sizes) and then ten graph-replayed steps.
+// steps (on a copy: search kernel, block sizes, chain or graph) and then ten
+// more in the way chosen.
 int trial_ms(const std::vector<HostState>& ms, double factor, double& ms_step, std::string& err) {
     std::vector<HostState> t = ms;
     for (HostState& m : t) regrid(m, factor);

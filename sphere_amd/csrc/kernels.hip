@@ -869,14 +869,19 @@ template <> struct PartnerVel<float> {
 };
 
 // Stores of what only the next step's own thread reads: springs and private
-// records.  In a system whose step moves more than the 256 MB that the
-// memory-side cache holds they would only push out of the caches what the step
-// still reads (its neighbours' records, the lists); below, the next step finds
-// them there.  us a step without and with: lattice of 262,144 spheres 50 and
-// 55, of 512,000 102 and 96, of 1,000,000 210 and 204; loose packing of 131,071
-// 36 and 39, of 400,000 89 and 88; crystal of 500,000 214 and 211, of 1,048,576
-// 429 and 426.  (Streaming their loads as well made the crystal slower: 473
-// against 450 a step, as stages.)
+// records.  In a system whose steps' state no longer fits the 256 MB of the
+// memory-side cache they would only push out of the caches what the step still
+// reads (its neighbours' records, the lists); below, the next step finds them
+// there.  us a step without and with: crystal of 171,500 spheres 59 and 73, of
+// 256,000 110 and 107, of 364,500 150 and 141, of 500,000 201 and 191, of
+// 1,048,576 398 and 382 (mixed precision 47 and 54, 68 and 83, 110 and 104, 150
+// and 146, 296 and 291); bonded 256,000 382 and 374; lattice of 262,144 51 and
+// 58, of 512,000 105 and 99, of 1,000,000 210 and 205; loose packing of 131,071
+// 36 and 38, of 300,000 61 and 73; ensemble of 328,596 66 and 75.  The line is
+// that of packings with few contacts, which lose most on the wrong side of it;
+// crystals pass it at about 240,000 spheres in FP64 and 330,000 in mixed
+// precision and lose up to 6 % below it.  (Streaming their loads as well made
+// the crystal slower: 473 against 450 a step, as stages.)
 constexpr uint32_t STREAM_NP = 400000;
 using nt4 = double __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void put(const DemDev& d, double4* p, double4 v) {
@@ -3120,7 +3125,7 @@ __device__ __forceinline__ uint32_t next_phase(const DemDev& d, uint32_t phase, 
 // one, whose search and force then run in one thread: the slot masks, the
 // particle's position and its slot words stay where the search left them, and
 // the force of one block hides the search of another.  us a step as stages and
-// as this chain: settling 990 spheres 47 and 16, 16,384 sheared 65 and 28,
+// as this chain: settling 990 spheres 47 and 16 (calls of 100 steps), 16,384 sheared 65 and 28,
 // 32,000 bonded 84 and 48; one lane a sphere: 131,072-sphere crystal 69 and 50,
 // 1,048,576 461 and 393 (mixed precision 363 and 293), loose packing of 131,071
 // under a moving wall 53 and 35, contact model 1 of 262,144 80 and 53; a
