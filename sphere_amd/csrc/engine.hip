@@ -1172,33 +1172,40 @@ int chained_steps(sph_dem* h, uint64_t n) {
 }
 
 // Chain or graph, for lists in a system too large for four lanes a sphere or
-// an ensemble, by the time of five steps each after three or four others.  The
-// chain wins where search and force are most of a step, the graph where most
-// steps sort or bonds are most of it: each stage then runs at its own
-// occupancy.  us a step as chain and as graph: crystal of 256,000 spheres 110
-// and 139, of 1,048,576 395 and 462; loose packing of 131,071 36 and 56, of
-// 300,000 61 and 80; lattice of 1,000,000 204 and 225; sheared 256,000 132 and
-// 160, 2,000,000 1,001 and 996; bonded 256,000 389 and 311; 64 calibration
+// an ensemble, by the time of four steps each after three or four others, the
+// shorter of two times (so that a list build in one of them does not decide).
+// The chain wins where search and force are most of a step, the graph where
+// most steps sort or bonds are most of it: each stage then runs at its own
+// occupancy.  us a step as chain and as graph: crystal of 256,000 spheres 109
+// and 139, of 1,048,576 396 and 461; loose packing of 131,071 36 and 55, of
+// 300,000 61 and 79; lattice of 1,000,000 204 and 226; sheared 256,000 132 and
+// 160, 2,000,000 1,001 and 996; bonded 256,000 388 and 305; 64 calibration
 // systems of 112,000 spheres 75 and 77, 512 of 8,464,166 1,930 and 1,610.
-// (The first step of a handle pays for it: crystal of 256,000 9.8 ms with it,
-// where 12.4 were taken by the trials of the stages alone while the copy of the
-// state was thirty-odd allocations.)
+// A tie goes to the chain, whose later steps gain on the graph's as spheres
+// move and lists are made (the lattice of 1,000,000: 205 and 199 in the trial);
+// with bonds to the graph (262,144 spheres: 398 and 380 in the trial, 335 and
+// 300 later).
+// (The first step of a handle pays for it: crystal of 256,000 10.9 ms with it,
+// where the trials of the stages alone took 12.4 while the copy of the state
+// was thirty-odd allocations.)
 int tune_chain(sph_dem* h) {
-    double ms[2];
+    double ms[2] = {HUGE_VAL, HUGE_VAL};
     for (int chain = 0; chain < 2; ++chain) {
         request_list_rebuild(h);
         // (the steps before make the lists and the graphs, or show how many
         // launches a step without new lists takes)
-        for (int part = chain ? 0 : 1; part < 3; ++part) {
+        for (int part = chain ? 0 : 1; part < 4; ++part) {
+            const uint64_t steps = part >= 2 ? 4 : chain ? 2 : 3;
             const auto t0 = std::chrono::steady_clock::now();
-            const int rc = chain ? chained_steps(h, part == 2 ? 5 : 2) : stage_steps(h, part == 2 ? 5 : 3);
+            const int rc = chain ? chained_steps(h, steps) : stage_steps(h, steps);
             if (rc) return rc;
-            ms[chain] = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+            const double t = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+            if (part >= 2) ms[chain] = std::min(ms[chain], t);
         }
     }
-    h->as_chain = ms[1] < ms[0];
+    h->as_chain = ms[1] < (h->hs.nb0 ? 1.0 : 1.04) * ms[0];
     if (h->verbosity > 1)
-        std::printf("sphere_dem: 5 steps as graph %.4f ms, as chain %.4f ms\n", ms[0], ms[1]);
+        std::printf("sphere_dem: 4 steps as graph %.4f ms, as chain %.4f ms\n", ms[0], ms[1]);
     return SPH_OK;
 }
 
