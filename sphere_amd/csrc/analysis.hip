@@ -1051,5 +1051,13 @@ extern "C" int sph_render(sph_t* h, int method, float max_val, float lower_cutof
         k_fill_u8<<<fill_blocks(bytes), ABLOCK, 0, h->stream>>>(img, bytes, 255);
     if (height > width) k_rt_repeat_rows<<<fill_blocks(bytes), ABLOCK, 0, h->stream>>>(img, width, height);
     A_TRY(hipGetLastError());
+    if (bytes > sph::GET_DIRECT && !s.p.empty()) {
+        // device memory allocated by this call: straight to the caller's (4,096
+        // spheres, 600 x 600 212 us through pinned slots and 166 this way,
+        // 800 x 800 249 and 207)
+        A_TRY(hipMemcpyAsync(rgb, img, bytes, hipMemcpyDeviceToHost, h->stream));
+        A_TRY(hipStreamSynchronize(h->stream));
+        return SPH_OK;
+    }
     return sph::copy_to_host(h, rgb, img, bytes);
 }

@@ -798,7 +798,7 @@ int download_all(sph_dem* h) {
 // take 39 us this way against 264 us for a copy into the caller's pageable
 // memory.  (Four threads sharing the copy out of the slots gained 1 % of 200
 // steps and four fields of 1,048,576 spheres.)
-constexpr size_t GET_DIRECT = 1 << 20, GET_SLOT = 2 << 20;
+constexpr size_t GET_DIRECT = sph::GET_DIRECT, GET_SLOT = 2 << 20;
 // (The control words lie in front of it: an allocation less at open.  Growing,
 // it keeps what it has until the new memory is there.)
 int get_pinned(sph_dem* h, size_t bytes) {
@@ -814,10 +814,12 @@ int get_pinned(sph_dem* h, size_t bytes) {
     return SPH_OK;
 }
 
-// A copy whose lines stay in the caches: the caller is likely to read them
-// next (a single large one goes past them -- positions of 60,000 spheres in
-// random order, read and set again, 848 us that way and 504 this; positions of
-// 1,048,576 and their mean 3.3 and 2.9 ms).
+// A copy whose lines stay in the caches, where the caller is likely to want
+// them next (one large memcpy goes past them).  us in one and in pieces:
+// positions of 60,000 spheres in random order read and set again 848 and 504,
+// of 195,112 2,390 and 1,400; of 300,763 and their mean 810 and 500, into memory
+// not touched before 2,520 and 2,000; of 1,030,301 and their mean 2,620 and
+// 1,940.
 void copy_out(char* dst, const char* src, size_t bytes) {
     constexpr size_t PIECE = 128 << 10;
     for (size_t k = 0; k < bytes; k += PIECE) std::memcpy(dst + k, src + k, std::min(PIECE, bytes - k));
@@ -1382,8 +1384,8 @@ std::vector<Comp> packed_comps(const sph::PState& p, int f) {
 
 // bytes from device memory to the caller's, behind what the stream holds:
 // through pinned memory in slots, the copy out of one beside the transfer into
-// another (two halves up to twice a slot: an image of 1.9 MB in one slot took
-// 277 us to the caller, in halves 253, as a plain copy 244).
+// another (two halves up to twice a slot: positions of 60,000 spheres 130 us
+// in one slot, 106 so and in copy_out's pieces).
 int sph::copy_to_host(sph_dem* h, void* dst, const void* src, size_t bytes) {
     const size_t slot = std::min(GET_SLOT, (bytes / 2 + 4095) / 4096 * 4096), slots = (bytes + slot - 1) / slot;
     int rc;

@@ -83,7 +83,7 @@ void enqueue_step(sph_dem* h, bool timed, int parity, bool lead, bool tail, bool
 
 // Device memory to the caller's, once the stream has come to this point.  Up
 // to GET_SMALL bytes it allocates nothing.
-constexpr size_t GET_SMALL = 64 << 10;
+constexpr size_t GET_SMALL = 64 << 10, GET_DIRECT = 1 << 20;
 int copy_to_host(sph_dem* h, void* dst, const void* src, size_t bytes);
 
 // Whether the handle's steps run as a chain of launches, and whether they can
