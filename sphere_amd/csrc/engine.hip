@@ -1185,8 +1185,9 @@ int chained_steps(sph_dem* h, uint64_t n) {
 // systems of 112,000 spheres 75 and 77, 512 of 8,464,166 1,930 and 1,610.
 // A tie goes to the chain, whose later steps gain on the graph's as spheres
 // move and lists are made (the lattice of 1,000,000: 205 and 199 in the trial);
-// with bonds to the graph (262,144 spheres: 398 and 380 in the trial, 335 and
-// 300 later).
+// with bonds or in an ensemble to the graph (bonded 262,144 spheres: 398 and
+// 380 in the trial, 335 and 300 later; the 512 systems in FP64 alike in the
+// trial, 1,690 and 1,550 later).
 // (The first step of a handle pays for it: crystal of 256,000 10.9 ms with it,
 // where the trials of the stages alone took 12.4 while the copy of the state
 // was thirty-odd allocations.)
@@ -1205,7 +1206,7 @@ int tune_chain(sph_dem* h) {
             if (part >= 2) ms[chain] = std::min(ms[chain], t);
         }
     }
-    h->as_chain = ms[1] < (h->hs.nb0 ? 1.0 : 1.04) * ms[0];
+    h->as_chain = ms[1] < (h->hs.nb0 || !h->members.empty() ? 1.0 : 1.04) * ms[0];
     if (h->verbosity > 1)
         std::printf("sphere_dem: 4 steps as graph %.4f ms, as chain %.4f ms\n", ms[0], ms[1]);
     return SPH_OK;
